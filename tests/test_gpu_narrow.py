@@ -12,6 +12,7 @@ import torch
 
 import knlp_amd as K
 from knlp_amd import _lib, ops
+from oracle import attention as A
 from tests import kvgen
 from tests.test_gpu_decode import _build, _check, _query, _run
 
@@ -168,3 +169,26 @@ def test_whole_row_shares(shape):
     _check(out, q, kp, vp, bt, lens, name=f"whole_rows_{name}")
     again = _run(q, kp, vp, bt, lens, hkv, d, split_tokens=0)
     assert torch.equal(out.view(torch.int16), again.view(torch.int16))
+
+
+# those whose other kernel is the VALU one, which sums in fp32
+FROM_VALU = [s for s in SHAPES if s[4] != s[5] or s[4] == 2 or (s[1] // s[2]) * (s[3] // s[7]) > 16]
+
+
+@pytest.mark.parametrize("shape", FROM_VALU, ids=lambda s: s[0])
+@pytest.mark.parametrize("split", [0, 128])
+def test_shapes_of_the_valu_kernel_keep_32_bit_sums(shape, split):
+    """An fp16 output differs from float64 by its own rounding (2e-4 of the
+    result here) and, beside it, by what 32-bit sums leave: 1e-5.  V codes as
+    fp16 subnormals lost 1.2e-4 in the matrix cores."""
+    name, hq, hkv, d, kf, vf, kgs, vgs = shape
+    lens = [1500, 700, 2100]
+    bt, kp, vp = _build(lens, hq, hkv, d, kf, vf, kgs, vgs, 80)
+    q = _query(len(lens), hq, d, 80)
+    out = _run(q, kp, vp, bt, lens, hkv, d, split_tokens=split).cpu().double().numpy()
+    ref = A.decode_reference_f64(q.float().numpy(), kp, vp, bt, lens)
+    norm = np.sqrt(np.mean(ref ** 2))
+    rounding = np.mean((ref.astype(np.float16).astype(np.float64) - ref) ** 2)
+    beside = np.sqrt(max(np.mean((out - ref) ** 2) - rounding, 0.0)) / norm
+    print(f"{name} {split}: {beside:.2e} beside a rounding of {np.sqrt(rounding) / norm:.2e}")
+    assert beside <= 1e-5
