@@ -86,7 +86,7 @@ Plane make_plane(PyObject* const* a, bool on_device) {
                               : fmt == KNLP_KV_INT8_SYM ? at::kChar : at::kByte;
   if (on_device) {
     require_device(r.data);
-    if (fmt != KNLP_KV_FP16) require_device(r.scales);
+    require_device(r.scales);
     if (fmt == KNLP_KV_INT4_ASYM) require_device(r.zeros);
   }
   TORCH_CHECK_VALUE(r.data.scalar_type() == want, "cache dtype ", r.data.scalar_type(),
@@ -290,6 +290,7 @@ PyObject* py_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const float scale = a[16] == Py_None ? static_cast<float>(1.0 / std::sqrt(static_cast<double>(d)))
                                        : static_cast<float>(real(a[16]));
   const int32_t dt = qs == at::kHalf ? KNLP_DT_F16 : KNLP_DT_BF16;
+  TORCH_CHECK_VALUE(slots || (!key && !value), "key and value need a slot_mapping");
   int32_t src = 0, sdt = 0;
   const float clip = static_cast<float>(real(a[22]));
   if (slots) {

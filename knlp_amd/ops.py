@@ -264,6 +264,8 @@ def append_and_decode(query, key, value, slot_mapping, key_cache, value_cache, k
     "fp16"; the caches, scales and zeros are the reference's tensors.  The
     written codes equal those of the separate append; the output equals the
     decode after it."""
+    if query.shape[0] and (slot_mapping is None or (key is None and value is None)):
+        raise ValueError("append_and_decode needs slot_mapping, and key or value")
     kf, vf = _fmt(k_format, asymmetric), _fmt(v_format, asymmetric)
     k = (key_cache, k_scales, k_zeros, kf,
          head_size if kf == KV_FP16 else (k_group_size or GROUP_SIZE))

@@ -64,3 +64,18 @@ def test_counts_reach_the_extension_as_integers(monkeypatch, kind):
     got = ops.fused_int4_decode(None, c, c, None, None, None, None, 8, 128,
                                 split_tokens=kind(128), total_context=kind(9000))
     assert got == (128, 9000) and all(type(n) is int for n in got)
+
+
+@pytest.mark.parametrize("rows,slots", [((1, 1), False), ((1, 0), False), ((0, 0), True),
+                                        ((0, 0), False)])
+def test_fused_append_needs_slots_and_rows(monkeypatch, rows, slots):
+    """A step without slots, or without any rows, is refused and not decoded
+    without its new token."""
+    monkeypatch.setattr(ops, "host", lambda: pytest.fail("the call reached the extension"))
+    q = torch.zeros(2, 8, 128, dtype=torch.float16)
+    c = torch.zeros(4, 16, 8, 64, dtype=torch.uint8)
+    s = torch.zeros(4, 16, 8, 4, dtype=torch.float16)
+    kv = [torch.zeros(2, 8, 128, dtype=torch.float16) if r else None for r in rows]
+    with pytest.raises(ValueError, match="slot_mapping"):
+        ops.append_and_decode(q, *kv, torch.zeros(2, dtype=torch.int64) if slots else None, c, c,
+                              s, s, None, None, 8, 128)
