@@ -145,7 +145,9 @@ def _run(query, k, v, block_size, block_table, seq_lens, num_kv_heads, head_size
          split_tokens, total_context, append=_NO_APPEND) -> torch.Tensor:
     """One decode; ``k`` and ``v`` are (cache, scales, zeros, format, group size)."""
     if split_tokens is None:
-        split_tokens = config.DECODE_SPLIT_TOKENS or -1           # -1: the library's schedule
+        split_tokens = config.DECODE_SPLIT_TOKENS or None
+    if split_tokens is None:
+        split_tokens = -1                                         # the library's schedule
     elif split_tokens < 0:
         raise ValueError("split_tokens must not be negative")
     return host().decode(query, *k, *v, block_size, block_table, seq_lens, num_kv_heads, head_size,

@@ -79,3 +79,21 @@ def test_fused_append_needs_slots_and_rows(monkeypatch, rows, slots):
     with pytest.raises(ValueError, match="slot_mapping"):
         ops.append_and_decode(q, *kv, torch.zeros(2, dtype=torch.int64) if slots else None, c, c,
                               s, s, None, None, 8, 128)
+
+
+def test_a_negative_split_is_refused_wherever_it_is_set(monkeypatch):
+    class Host:
+        @staticmethod
+        def decode(*a):
+            return a[17]
+    monkeypatch.setattr(ops, "host", lambda: Host)
+    c = torch.zeros(4, 16, 8, 64, dtype=torch.uint8)
+    args = (None, c, c, None, None, None, None, 8, 128)
+    for setting, want in ((0, -1), (256, 256)):                  # 0: the library's schedule
+        monkeypatch.setattr(ops.config, "DECODE_SPLIT_TOKENS", setting)
+        assert ops.fused_int4_decode(*args) == want
+    with pytest.raises(ValueError, match="negative"):
+        ops.fused_int4_decode(*args, split_tokens=-64)
+    monkeypatch.setattr(ops.config, "DECODE_SPLIT_TOKENS", -64)
+    with pytest.raises(ValueError, match="negative"):
+        ops.fused_int4_decode(*args)
