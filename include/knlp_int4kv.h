@@ -149,13 +149,23 @@ int32_t knlp_kv_decode_plan(int32_t num_seqs, int32_t num_kv_heads,
  * kernel takes besides (kv heads in fours or twos; fp16 K with 16 < G groups
  * <= 32) that kernel's own: 0 (stream) for a variable-length batch, else a
  * split length.  Same arguments and result as knlp_kv_decode_plan; a caller
- * of either may pass its result to any decode entry point.
+ * of either may pass its result to any decode entry point.  The answer is the
+ * shape's: where the planes turn out not to lie as that kernel needs them, a
+ * stream schedule is run as split-K inside its workspace, with splits sized by
+ * that.  knlp_kv_decode_schedule_planes looks at the planes and the page size
+ * and answers with the plan for those.
  */
 int32_t knlp_kv_decode_schedule(int32_t num_seqs, int32_t num_kv_heads,
                                 int32_t num_q_heads, int32_t head_size,
                                 int32_t max_context, int64_t total_context,
                                 int32_t k_format, int32_t k_group_size,
                                 int32_t v_format, int32_t v_group_size);
+
+int32_t knlp_kv_decode_schedule_planes(int32_t num_seqs, int32_t num_kv_heads,
+                                       int32_t num_q_heads, int32_t head_size,
+                                       int32_t max_context, int64_t total_context,
+                                       const knlp_kv_plane* key_cache,
+                                       const knlp_kv_plane* value_cache, int32_t block_size);
 
 /* Bytes of fp32 workspace decode needs for this shape and split length
  * (split_tokens = 0: the stream schedule's). */

@@ -24,7 +24,7 @@ KV_INT4_SYM, KV_INT4_ASYM, KV_INT8_SYM, KV_FP16 = 0, 1, 2, 3
 EXPORTS = (
     "knlp_abi_version", "knlp_status_string", "knlp_kv_append",
     "knlp_kv_decode_split_tokens", "knlp_kv_decode_plan", "knlp_kv_decode_schedule",
-    "knlp_kv_decode_workspace_bytes",
+    "knlp_kv_decode_schedule_planes", "knlp_kv_decode_workspace_bytes",
     "knlp_kv_decode_partial", "knlp_kv_decode_merge", "knlp_kv_decode",
     "knlp_kv_decode_kernel_kind", "knlp_kv_append_decode", "knlp_int4_twos_to_offset",
     "knlp_kv_decode_noalloc", "knlp_hbm_read_probe", "knlp_prefill_attention",
@@ -63,6 +63,8 @@ _SIGS = {
     "knlp_kv_decode_plan": (_I32, [_I32, _I32, _I32, _I32, _I32, _I64, _I32, _I32, _I32, _I32]),
     "knlp_kv_decode_schedule": (_I32, [_I32, _I32, _I32, _I32, _I32, _I64, _I32, _I32, _I32,
                                        _I32]),
+    "knlp_kv_decode_schedule_planes": (_I32, [_I32, _I32, _I32, _I32, _I32, _I64, _PLANE, _PLANE,
+                                              _I32]),
     "knlp_kv_decode_workspace_bytes": (_I64, [_I32, _I32, _I32, _I32, _I32]),
     "knlp_kv_decode_partial": (_I32, [_P, _I32, _I64, _I64, _I32, _I32, _I32, _I32,
                                       _PLANE, _PLANE, _P, _I64, _P, _I32, _I32, _F, _I32,

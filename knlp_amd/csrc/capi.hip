@@ -288,6 +288,24 @@ int32_t knlp_kv_decode_schedule(int32_t num_seqs, int32_t num_kv_heads, int32_t 
   return static_cast<int32_t>(std::min(std::max<int64_t>((t + tile - 1) / tile, 1) * tile, most));
 }
 
+int32_t knlp_kv_decode_schedule_planes(int32_t num_seqs, int32_t num_kv_heads,
+                                       int32_t num_q_heads, int32_t head_size,
+                                       int32_t max_context, int64_t total_context,
+                                       const knlp_kv_plane* key_cache,
+                                       const knlp_kv_plane* value_cache, int32_t block_size) {
+  if (key_cache == nullptr || value_cache == nullptr) return KNLP_ERR_ARG;
+  DecodeArgs a{};
+  a.kp = fp16_groups_as_rows(*key_cache, head_size);
+  a.vp = fp16_groups_as_rows(*value_cache, head_size);
+  a.num_kv_heads = num_kv_heads;
+  a.group = num_kv_heads > 0 ? num_q_heads / num_kv_heads : 0;
+  a.block_size = block_size;
+  const auto answer = coop_extra_supported(a, head_size) ? knlp_kv_decode_schedule
+                                                         : knlp_kv_decode_plan;
+  return answer(num_seqs, num_kv_heads, num_q_heads, head_size, max_context, total_context,
+                a.kp.format, a.kp.group_size, a.vp.format, a.vp.group_size);
+}
+
 int32_t knlp_kv_decode_split_tokens(int32_t num_seqs, int32_t num_kv_heads, int32_t num_q_heads,
                                     int32_t head_size, int32_t max_context, int32_t k_format,
                                     int32_t v_format) {
@@ -422,9 +440,7 @@ int decode_partial(const void* query, int32_t q_dtype, int64_t q_stride_seq,
   hipStream_t hs = static_cast<hipStream_t>(stream_ptr);
   // (any finite softmax scale: the matrix-core kernels fold a negative one's
   // sign into q and treat 0 as uniform weights)
-  // (16-token sub-tiles inside one page)
-  const int extra = block_size >= 16 && is_pow2(block_size)
-                        ? coop_extra_supported(a, head_size) : 0;
+  const int extra = coop_extra_supported(a, head_size);
   const bool mfma = kind == 1 && mfma_layout_ok(kp, head_size, block_size) &&
                     mfma_layout_ok(vp, head_size, block_size);
   int32_t* fallback_hdr = nullptr;

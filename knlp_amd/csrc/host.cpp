@@ -274,14 +274,11 @@ PyObject* py_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     "key and value caches have different block sizes");
   const int64_t max_context = table.size(1) * block_size;
   if (split < 0) {
-    // (the kernels that the schedule plans for besides the plan's take pages of
-    // 16 tokens or more)
-    const bool pages = block_size >= 16 && (block_size & (block_size - 1)) == 0;
-    split = (pages ? knlp_kv_decode_schedule : knlp_kv_decode_plan)(
+    split = knlp_kv_decode_schedule_planes(
         static_cast<int32_t>(seqs), static_cast<int32_t>(hkv), static_cast<int32_t>(hq),
-        static_cast<int32_t>(d), static_cast<int32_t>(max_context), total, kp.p.format,
-        kp.p.group_size, vp.p.format, vp.p.group_size);
-    check_status(split, "knlp_kv_decode_schedule");
+        static_cast<int32_t>(d), static_cast<int32_t>(max_context), total, &kp.p, &vp.p,
+        block_size);
+    check_status(split, "knlp_kv_decode_schedule_planes");
   }
   const int64_t ws_bytes = knlp_kv_decode_workspace_bytes(
       static_cast<int32_t>(seqs), static_cast<int32_t>(hq), static_cast<int32_t>(d),

@@ -168,7 +168,7 @@ int launch_merge(const float* part_o, const float* part_ml, const int32_t* seq_l
                  hipStream_t stream, const int32_t* stream_meta = nullptr,
                  const int32_t* stream_hdr = nullptr);
 // shapes that only the cooperative kernel's further instances take (0: not
-// one), with and without their planes' layouts, and their launch
+// one), without and with their planes' layouts, and their launch
 int coop_extra_parts(int num_kv_heads, int group, int head_size, int k_format, int k_gs,
                      int v_format, int v_gs);
 int coop_extra_supported(const DecodeArgs& a, int head_size);

@@ -339,6 +339,52 @@ def test_schedule_is_the_plan_where_no_layout_fits_the_narrow_kernels():
         assert L.knlp_kv_decode_schedule(8, hkv, hq, d, 4096, 0, *fmt) == 0
 
 
+def _rows_plane(fmt, hkv, d, gs, page=16, room=0, apart=1):
+    """A plane of hkv heads, cut out of one of hkv + room, every `apart`-th one."""
+    row = d if fmt in (_lib.KV_FP16, _lib.KV_INT8_SYM) else d // 2
+    h, p = (hkv + room) * apart, _lib.KvPlane()
+    p.format, p.group_size, p.data = fmt, gs, 0x1000
+    p.stride_head, p.stride_page, p.stride_block = row * apart, h * row, page * h * row
+    if fmt != _lib.KV_FP16:
+        ng = d // gs
+        p.scales, p.zeros = 0x10000, 0x20000
+        for x in "sz":
+            for k, v in (("head", ng * apart), ("page", h * ng), ("block", page * h * ng)):
+                setattr(p, f"{x}_stride_{k}", v)
+    return p
+
+
+@pytest.mark.parametrize("hq,hkv,d,kf,kgs,vf,vgs", [
+    (14, 2, 64, _lib.KV_INT4_ASYM, 32, _lib.KV_INT4_ASYM, 32),
+    (28, 4, 128, _lib.KV_INT8_SYM, 32, _lib.KV_INT4_SYM, 32),
+    (28, 4, 128, _lib.KV_FP16, 128, _lib.KV_INT4_ASYM, 32),
+    (32, 8, 128, _lib.KV_INT4_ASYM, 32, _lib.KV_INT4_ASYM, 32)])
+def test_schedule_of_planes_is_the_plan_on_other_layouts(hq, hkv, d, kf, kgs, vf, vgs):
+    """Dense pages of 16 tokens or a larger power of two: the schedule; heads
+    with gaps between them, scales of a token under 16 bytes in a wider cache
+    and pages of 8 or 24 tokens run on the other kernels: the plan's split."""
+    L = _lib.lib()
+    other = [(dict(apart=2), {}), ({}, dict(apart=2)), (dict(page=8), dict(page=8)),
+             (dict(page=24), dict(page=24))]
+    if d == 64:
+        other.append((dict(room=2), dict(room=2)))
+    fmt = (kf, kgs, vf, vgs)
+    for S, total in ((8, 0), (8, 9000), (8, 32768), (1, 0)):
+        shape = (S, hkv, hq, d, 4096, total)
+
+        def planes(k, v):
+            return L.knlp_kv_decode_schedule_planes(
+                *shape, ctypes.byref(_rows_plane(kf, hkv, d, kgs, **k)),
+                ctypes.byref(_rows_plane(vf, hkv, d, vgs, **v)), k.get("page", 16))
+        plan = L.knlp_kv_decode_plan(*shape, *fmt)
+        assert planes({}, {}) == planes(dict(page=64), dict(page=64)) == \
+            L.knlp_kv_decode_schedule(*shape, *fmt)
+        for k, v in other:
+            assert planes(k, v) == plan, (S, total, k, v)
+        assert plan > 0 or hkv == 8
+    assert L.knlp_kv_decode_schedule_planes(8, hkv, hq, d, 4096, 0, None, None, 16) == _lib.ERR_ARG
+
+
 @no_gpu_only
 def test_stream_fallback_shape_error_comes_before_any_launch():
     """The stream schedule (split 0) on planes only split-K takes falls back to
