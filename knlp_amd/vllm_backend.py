@@ -44,6 +44,7 @@ from typing import ClassVar
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from vllm.logger import init_logger
 from vllm.v1.attention.backend import (
@@ -68,6 +69,14 @@ DECODE_KERNELS = {
     ("fp16", "int4"): "kfp16_vint4_decode",
     ("fp16", "int8"): "kfp16_vint8_decode",
 }
+
+
+def _differentiated(*tensors) -> bool:
+    """Whether a call on these tensors (or None) has a gradient to record or
+    carries a forward-mode tangent, which the kernels would drop."""
+    ts = [t for t in tensors if t is not None]
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in ts)) or \
+        any(forward_ad.unpack_dual(t).tangent is not None for t in ts)
 
 
 @dataclass
@@ -233,7 +242,9 @@ class FusedInt4AttentionImpl(AttentionImpl[FusedInt4AttentionMetadata]):
     def _copies_bits(self, key, value, key_cache, value_cache, slot_mapping) -> bool:
         """Whether these bf16 rows and planes can go through the append
         kernel's row copy: device tensors of one layout, heads it takes, rows
-        on its 4-byte grid."""
+        on its 4-byte grid, nothing to differentiate."""
+        if _differentiated(key, value, key_cache, value_cache):
+            return False
         if not (key_cache.is_cuda and slot_mapping.is_cuda and slot_mapping.dim() == 1 and
                 slot_mapping.dtype in (torch.int32, torch.int64) and
                 self.head_size in (32, 64, 128, 256)):
@@ -479,10 +490,9 @@ class FusedInt4AttentionImpl(AttentionImpl[FusedInt4AttentionMetadata]):
     def _prefill_fused(self, query, key, value, qsl, output) -> bool:
         """Causal attention of the batch's prompts of two tokens or more in
         one launch (ops.prefill_attention); False, with nothing done, for
-        tensors that the kernel does not take, positions on the host or a
-        gradient to record."""
-        if qsl.device != query.device or (torch.is_grad_enabled() and
-                                          any(t.requires_grad for t in (query, key, value))):
+        tensors that the kernel does not take, positions on the host, a
+        gradient to record or a forward-mode tangent to carry."""
+        if qsl.device != query.device or _differentiated(query, key, value, output):
             return False
         k3 = key.view(-1, self.num_kv_heads, self.head_size) if key.dim() == 2 else key
         v3 = value.view(-1, self.num_kv_heads, self.head_size) if value.dim() == 2 else value

@@ -302,3 +302,18 @@ def test_prefill_route(vb, monkeypatch, case):
     want = causal_ref(q, k, v, lens)
     got = out.detach().float().cpu().numpy().reshape(-1)
     assert close(got, torch.as_tensor(want).float().numpy().reshape(-1))
+
+
+def test_bf16_paged_write_records_a_gradient(vb, monkeypatch):
+    """Rows with a gradient to record go through the scatter, which records it."""
+    impl = impl_for(vb, monkeypatch)
+    key, value = (torch.randn(3, HKV, D).bfloat16().cuda().requires_grad_(r) for r in (1, 0))
+    kv = torch.zeros(2, NB, BS, HKV, D, dtype=torch.bfloat16, device="cuda")
+    slots = torch.tensor([5, -1, 17], device="cuda")
+    assert not impl._copies_bits(key, value, kv[0], kv[1], slots)
+    with torch.no_grad():
+        assert impl._copies_bits(key, value, kv[0], kv[1], slots)
+    kc = kv[0].clone()
+    impl._write_paged_fp16(key, value, kc, kv[1], slots)
+    kc.float().sum().backward()
+    assert key.grad is not None and float(key.grad.float().sum()) == 2 * HKV * D

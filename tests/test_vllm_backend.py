@@ -354,3 +354,29 @@ def test_warmup_without_metadata(vb, monkeypatch):
     o = torch.ones_like(q)
     assert impl.forward(None, q, q, q, torch.empty(0), decode_md(vb, [1], [0]), output=o) is o
     assert float(o.abs().sum()) == 0.0
+
+
+@pytest.mark.parametrize("which", ["query", "key", "value", "output", None])
+@pytest.mark.parametrize("mode", ["gradient", "tangent"])
+def test_prefill_kernel_leaves_differentiated_calls_to_sdpa(vb, monkeypatch, which, mode):
+    """A recorded gradient or a forward-mode tangent of any operand goes down
+    the per-prompt path, which carries it; the kernel would drop it."""
+    from torch.autograd import forward_ad
+    impl = vb.FusedInt4AttentionImpl(4, 64, 0.125, num_kv_heads=2)
+    launched = []
+    monkeypatch.setattr(vb.ops, "prefill_supported", lambda *a: True)
+    monkeypatch.setattr(vb.ops, "prefill_attention", lambda *a, **k: launched.append(a))
+    t = dict(query=torch.randn(5, 4, 64), key=torch.randn(5, 2, 64), value=torch.randn(5, 2, 64),
+             output=torch.zeros(5, 256))
+    qsl = torch.tensor([0, 2, 5], dtype=torch.int32)
+    with forward_ad.dual_level():
+        if which and mode == "gradient":
+            t[which].requires_grad_()
+        elif which:
+            t[which] = forward_ad.make_dual(t[which], torch.ones_like(t[which]))
+        done = impl._prefill_fused(t["query"], t["key"], t["value"], qsl, t["output"])
+        assert done == bool(launched) == (which is None)
+        if mode == "tangent" and which in ("query", "key", "value"):
+            impl._prefill_rows(t["query"], t["key"], t["value"], qsl, torch.arange(2),
+                               t["output"])
+            assert forward_ad.unpack_dual(t["output"]).tangent.abs().sum() > 0
