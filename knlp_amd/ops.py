@@ -29,7 +29,6 @@ kernels pick their own token tiles.
 from __future__ import annotations
 
 import ctypes
-import math
 
 import torch
 
@@ -164,9 +163,10 @@ def _decode(query, kp: KvPlane, vp: KvPlane, block_size, block_table, seq_lens, 
 def prefill_supported(query, key, value, out, scale) -> bool:
     """Whether :func:`prefill_attention` takes these tensors: device tensors of
     one 16-bit dtype, heads of 64 or 128, rows that 16-byte loads can read, K
-    and V rows in order."""
+    and V rows in order, an output apart from them (its rows are written while
+    other blocks still read), a scale that is finite in fp32 (None: 1/sqrt(D))."""
     if not (query.is_cuda and query.dtype in _SRC_DTYPES and query.dim() == 3 and
-            query.shape[2] in (64, 128) and math.isfinite(scale)):
+            query.shape[2] in (64, 128) and (scale is None or abs(scale) < 2.0 ** 127)):
         return False
     for t in (query, key, value, out):
         if (t.dim() != 3 or t.dtype != query.dtype or t.device != query.device or
@@ -175,6 +175,11 @@ def prefill_supported(query, key, value, out, scale) -> bool:
             return False
     if not all(query.shape[2] <= t.stride(0) < 1 << 24 for t in (key, value)):
         return False                       # repeated or overlapping rows
+    if any(_same_storage(out, t) for t in (key, value)):
+        return False
+    if _same_storage(out, query) and (out.data_ptr() != query.data_ptr() or
+                                      out.stride() != query.stride()):
+        return False                       # (in place: a block reads only the rows it writes)
     return (out.shape[1] == query.shape[1] and key.shape[1] == value.shape[1] > 0 and
             query.shape[1] % key.shape[1] == 0)
 

@@ -97,3 +97,31 @@ def test_a_negative_split_is_refused_wherever_it_is_set(monkeypatch):
     monkeypatch.setattr(ops.config, "DECODE_SPLIT_TOKENS", -64)
     with pytest.raises(ValueError, match="negative"):
         ops.fused_int4_decode(*args)
+
+
+class _OnDevice:
+    """A CPU tensor that says it is a device tensor (nothing is launched)."""
+    is_cuda = True
+
+    def __init__(self, t):
+        self._t = t
+
+    def __getattr__(self, name):
+        return getattr(self._t, name)
+
+
+def test_prefill_kernel_takes_no_overlapping_output_or_odd_scale():
+    """An output in K's or V's memory would be written while other blocks read
+    it; a scale of None is the default and one beyond fp32 is not taken."""
+    rows = torch.zeros(4, 6, 64, dtype=torch.float16)
+    q, k, v = (_OnDevice(torch.zeros(4, h, 64, dtype=torch.float16)) for h in (6, 6, 6))
+    out = _OnDevice(rows)
+    for scale, ok in ((0.1, True), (None, True), (-3.0, True), (1e39, False),
+                      (float("inf"), False), (float("nan"), False)):
+        assert ops.prefill_supported(q, k, v, out, scale) == ok, scale
+    assert not ops.prefill_supported(q, out, v, out, 0.1)
+    assert not ops.prefill_supported(q, k, out, out, 0.1)
+    assert ops.prefill_supported(out, k, v, out, 0.1)      # a block reads only the q rows it writes
+    shifted = _OnDevice(torch.zeros(5, 6, 64, dtype=torch.float16)[1:])
+    before = _OnDevice(torch.as_strided(shifted._t, (4, 6, 64), (384, 64, 1), 0))
+    assert not ops.prefill_supported(shifted, k, v, before, 0.1)
