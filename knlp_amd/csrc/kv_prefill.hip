@@ -65,6 +65,7 @@ constexpr int kWaves = 4;
 // (log2 units), so p <= 4 and p 2^12 <= 2^14, inside fp16
 constexpr float kRaise = 2.0f;
 constexpr float kPScale = 12.0f;
+constexpr float kBaseMax = 1024.0f;
 
 template <bool BF16>
 __device__ __forceinline__ f16x mfma(u4 a, u4 b, f16x c) {
@@ -302,7 +303,18 @@ void prefill_kernel(PrefillArgs a) {
       }
       // p = 2^(12 + (score - max) sl2), the max's part taken out once (every
       // score so far -inf: any finite base gives p = 0)
-      const float base = kPScale - (m_run == -INFINITY ? 0.0f : m_run) * sl2;
+      const float ref = m_run == -INFINITY ? 0.0f : m_run;
+      float base = kPScale - ref * sl2;
+      // the base is rounded to its own last bit, which is part of p's exponent:
+      // where that grows past 2^-14 the max is taken from the scores instead
+      if (__any(fabsf(base) > kBaseMax)) {       // uniform, rare
+        asm volatile("");                        // (a branch, as above)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[x][r] -= ref;
+        base = kPScale;
+      }
       uint32_t hi[16], lo[16];
 #pragma unroll
       for (int x = 0; x < 2; ++x)

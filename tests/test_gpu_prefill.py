@@ -115,6 +115,26 @@ def test_prefill_peaked_and_flat_rows():
         check(out, reference(q, keys, v, [n], d ** -0.5), v, torch.float16)
 
 
+@pytest.mark.parametrize("dtype,big", [(torch.float16, 2.0 ** 5), (torch.float16, 2.0 ** 15),
+                                       (torch.bfloat16, 2.0 ** 40)])
+def test_prefill_scores_of_any_size(dtype, big):
+    """Scores far beyond 2^24 (exact: one dimension, whole multiples of a power
+    of two): the largest so far takes the whole row, two equal ones share it.
+    With a scale of 1 the softmax's max in its log2 units has no bits left for
+    an exponent of p beside it."""
+    n, d = 300, 128
+    g = torch.Generator().manual_seed(8)
+    rank = torch.randperm(n, generator=g) // 2                    # each value twice
+    v = torch.randn(n, 1, d, generator=g).to(dtype)
+    q, k = torch.zeros(n, 1, d), torch.zeros(n, 1, d)
+    q[:, 0, 3] = big
+    k[:, 0, 3] = (rank - 75) * (big / 256)
+    q, k = q.to(dtype), k.to(dtype)
+    out = torch.zeros(n, 1, d, dtype=dtype, device="cuda")
+    K.prefill_attention(q.cuda(), k.cuda(), v.cuda(), starts([n]), out, scale=1.0)
+    check(out, reference(q, k, v, [n], 1.0), v, dtype)
+
+
 def test_prefill_unsupported_tensors_raise():
     q = torch.zeros(4, 2, 128, dtype=torch.float16, device="cuda")
     qsl = starts([4])

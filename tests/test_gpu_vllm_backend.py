@@ -307,7 +307,7 @@ def test_prefill_route(vb, monkeypatch, case):
 def test_bf16_paged_write_records_a_gradient(vb, monkeypatch):
     """Rows with a gradient to record go through the scatter, which records it."""
     impl = impl_for(vb, monkeypatch)
-    key, value = (torch.randn(3, HKV, D).bfloat16().cuda().requires_grad_(r) for r in (1, 0))
+    key, value = (torch.randn(3, HKV, D).bfloat16().cuda().requires_grad_(r) for r in (True, False))
     kv = torch.zeros(2, NB, BS, HKV, D, dtype=torch.bfloat16, device="cuda")
     slots = torch.tensor([5, -1, 17], device="cuda")
     assert not impl._copies_bits(key, value, kv[0], kv[1], slots)
