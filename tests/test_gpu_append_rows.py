@@ -1,9 +1,11 @@
 """The append kernel's branches, bit for bit against the oracle: one row and
-four rows per thread (65536 (token, head) rows is the line) with remainders,
-wide and narrow loads and stores (rows off the 16-byte and 4-byte grid), page
+four rows per thread (from kBulkRows (token, head) rows on) with remainders, wide and narrow loads and stores (rows off the 16-byte and 4-byte grid), page
 sizes that are no power of two, groups so large or small that the quotients
 are divided instead of taken through the reciprocal, and values on the
 rounding thresholds of their group."""
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -14,6 +16,8 @@ from tests import kvgen
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+with open(os.path.join(os.path.dirname(K.__file__), "csrc", "kv_append.hip")) as f:
+    LINE = int(re.search(r"kBulkRows = (\d+);", f.read())[1])
 
 
 def rows(n, hkv, d, seed, dtype, shift=0):
@@ -73,11 +77,26 @@ def check(fmt, tokens, hkv, d, gs, page, dtype, shift, code_shift, clip=10.0):
 
 
 @pytest.mark.parametrize("fmt", ["int4_asym", "int4_sym", "int8"])
-@pytest.mark.parametrize("tokens,hkv,d,gs", [(8191, 8, 128, 32), (8192, 8, 64, 16),
-                                             (9363, 7, 128, 128), (1, 3, 32, 32),
+@pytest.mark.parametrize("tokens,hkv,d,gs", [(LINE // 8 - 1, 8, 32, 32), (LINE // 8, 8, 64, 16),
+                                             (LINE // 7 + 1, 7, 32, 16), (LINE // 4 + 5, 4, 128, 128),
+                                             (LINE // 4 + 1, 4, 256, 64), (1, 3, 32, 32),
                                              (67, 5, 256, 64)])
 def test_rows_per_thread(fmt, tokens, hkv, d, gs):
+    """Below the line, on it, and past it with a last block of few rows."""
     check(fmt, tokens, hkv, d, gs, 16, torch.float16, 0, 0)
+
+
+def test_four_rows_per_thread_copy_fp16_and_take_unaligned_rows():
+    n, hkv, d = LINE // 4 + 3, 4, 64
+    for shift in (0, 2):
+        k = rows(n, hkv, d, 7, torch.float16, shift)
+        cache = torch.zeros(n // 16 + 2, 16, hkv, d, dtype=torch.float16, device=DEV)
+        slots = torch.randperm(n + 16, generator=torch.Generator().manual_seed(6))[:n].to(DEV)
+        K.reshape_and_cache_fp16(k, None, cache, None, slots)
+        want = torch.zeros((n // 16 + 2) * 16, hkv, d, dtype=torch.float16, device=DEV)
+        want[slots] = k
+        assert torch.equal(cache.view_as(want), want)
+    check("int4_asym", LINE // 8 + 1, 8, 32, 32, 24, torch.bfloat16, 2, 4)
 
 
 @pytest.mark.parametrize("fmt,code_shifts", [("int4_asym", (0, 1, 4)), ("int4_sym", (2, 3)),

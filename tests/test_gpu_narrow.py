@@ -47,6 +47,9 @@ SHAPES = [
 LENS = [1, 31, 32, 33, 63, 64, 65, 96, 127, 128, 129, 0, 700, 1025, 2100]
 
 
+TILE = {2: 128, 6: 128}            # tokens of a tile by kv heads, else 64
+
+
 def planned(hq, hkv, d, kf, vf, kgs, vgs):
     """knlp_kv_decode_schedule answers for the shape where the plan does not."""
     L = _lib.lib()
@@ -68,15 +71,20 @@ def test_narrow_matches_oracle(shape, split):
 
 
 @pytest.mark.parametrize("split", [0, 128])
-@pytest.mark.parametrize("shape", [s for s in SHAPES if s[4] != 3], ids=lambda s: s[0])
-def test_narrow_fused_append(shape, split):
+@pytest.mark.parametrize("shape,sides", [(s, "kv") for s in SHAPES] +
+                         [(s, "v") for s in SHAPES if s[4] == 3],
+                         ids=lambda x: x if isinstance(x, str) else x[0])
+def test_narrow_fused_append(shape, sides, split):
     """The new token's rows written by the decode launch: the codes of the
-    separate append and the decode that follows it, bit for bit."""
+    separate append and the decode that follows it, bit for bit.  (fp16 K also
+    with its row already in the cache.)"""
     name, hq, hkv, d, kf, vf, kgs, vgs = shape
     lens = [1, 32, 33, 64, 129, 600]
     bt, kp, vp = _build(lens, hq, hkv, d, kf, vf, kgs, vgs, 40)
     q = _query(len(lens), hq, d, 41).to(DEV)
     new = [kvgen.randn((len(lens), hkv, d), s, torch.float16).to(DEV) for s in (42, 43)]
+    if sides == "v":
+        new[0] = None
     pos = np.array(lens) - 1
     slots = torch.from_numpy(bt[np.arange(len(lens)), pos // 16].astype(np.int64) * 16 + pos % 16)
     sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
@@ -88,11 +96,12 @@ def test_narrow_fused_append(shape, split):
         planes = (ops._plane(kd, ks, kz, kf, kgs), ops._plane(vd, vs, vz, vf, vgs))
         args = (new[0], new[1], slots.to(DEV), 10.0)
         if not fused:
-            ops._append(new[0], new[1], *planes, slots.to(DEV), 10.0, 16)
+            ops._append(new[0], new[1], planes[0] if sides == "kv" else None, planes[1],
+                        slots.to(DEV), 10.0, 16)
         out = ops._decode(q, *planes, 16, btd, sl, hkv, d, split_tokens=split,
                           append=args if fused else None)
         torch.cuda.synchronize()
-        outs.append([out, kd, vd, ks, vs] + [t for t in (kz, vz) if t is not None])
+        outs.append([t for t in (out, kd, vd, ks, vs, kz, vz) if t is not None])
     for a, b in zip(*outs):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), name
 
@@ -168,6 +177,41 @@ def test_whole_row_shares(shape):
     out = _run(q, kp, vp, bt, lens, hkv, d, split_tokens=0)
     _check(out, q, kp, vp, bt, lens, name=f"whole_rows_{name}")
     again = _run(q, kp, vp, bt, lens, hkv, d, split_tokens=0)
+    assert torch.equal(out.view(torch.int16), again.view(torch.int16))
+
+
+@pytest.mark.parametrize("charged", [False, True])
+@pytest.mark.parametrize("shape", [SHAPES[i] for i in (0, 3, 5, 9, 12, 14, 17, 19)],
+                         ids=lambda s: s[0])
+def test_several_segments_in_a_block(shape, charged):
+    """A batch of more rows than a quarter of the CUs and more tiles than CUs:
+    equal shares, with the charge of 6 tiles a row from 7 tiles a CU on, so
+    most blocks end one row and start another: partials, their combination and
+    the next row's copies in the same LDS.  (All sequences draw on one small
+    pool of pages.)"""
+    name, hq, hkv, d, kf, vf, kgs, vgs = shape
+    tile = 32 if kf == 3 else TILE.get(hkv, 64)
+    heads = 4 if kf == 3 or hkv % 4 == 0 else 2
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    seqs, nhg, bs = 96, hkv // heads, 16
+    g = np.random.default_rng(len(name) + charged)
+    lens = [int(n) for n in g.integers(1, (44 if charged else 9) * tile // nhg, seqs)]
+    lens[3], lens[7], lens[8] = 0, 1, tile + 1
+    tiles = nhg * sum(-(-n // tile) for n in lens)
+    rows = nhg * sum(n > 0 for n in lens)
+    assert 4 * rows > cus and (tiles >= 7 * cus if charged else cus < tiles < 7 * cus)
+    nb = 200
+    table = g.integers(0, nb, (seqs, -(-max(lens) // bs))).astype(np.int32)
+    planes = []
+    for f, gs, seed in ((kf, kgs, 1), (vf, vgs, 2)):
+        p = kvgen.empty_plane(f, nb, bs, hkv, d, gs)
+        kvgen.fill_plane(p, kvgen.randn((nb * bs, hkv, d), seed, outlier_frac=0.01).float().numpy(),
+                         np.arange(nb * bs))
+        planes.append(p)
+    q = _query(seqs, hq, d, 90)
+    out = _run(q, *planes, table, lens, hkv, d, split_tokens=0)
+    _check(out, q, *planes, table, lens, name=f"segments_{name}_{charged}")
+    again = _run(q, *planes, table, lens, hkv, d, split_tokens=0)
     assert torch.equal(out.view(torch.int16), again.view(torch.int16))
 
 

@@ -65,6 +65,24 @@ def test_prefill_any_finite_scale(scale):
     check(out, reference(q, k, v, [150], scale), v, torch.float16)
 
 
+@pytest.mark.parametrize("seqs", [64, 65, 130])
+def test_prefill_of_many_short_prompts(seqs):
+    """Up to 64 sequences the tiles of all go longest first; past that they are
+    laid end to end, 64 at a time.  Empty sequences and one-token rows (left
+    out, min_len = 2) among them, and two tiles in some."""
+    g = torch.Generator().manual_seed(seqs)
+    lens = torch.randint(0, 40, (seqs,), generator=g).tolist()
+    lens[5], lens[6], lens[-1], lens[seqs // 2] = 0, 1, 200, 129
+    n, hq, hkv, d = sum(lens), 4, 2, 64
+    q, k, v = (torch.randn(n, h, d, generator=g).half() for h in (hq, hkv, hkv))
+    out = torch.full((n, hq, d), 7.0, dtype=torch.float16, device="cuda")
+    K.prefill_attention(q.cuda(), k.cuda(), v.cuda(), starts(lens), out, min_len=2)
+    ref = reference(q, k, v, lens, d ** -0.5)
+    one = torch.repeat_interleave(torch.tensor(lens), torch.tensor(lens)) == 1
+    assert bool((out.cpu()[one] == 7.0).all()) and bool(one.any())
+    check(out.cpu()[~one], ref[~one], v, torch.float16)
+
+
 def test_prefill_strided_rows_and_short_rows_left_out():
     """q, k, v as views of one fused qkv tensor, an output with other rows
     around it, and the batch's one-token rows not written (min_len = 2)."""
