@@ -148,7 +148,11 @@ int32_t knlp_kv_decode_plan(int32_t num_seqs, int32_t num_kv_heads,
  * above where it covers the shape, and for dense caches that the cooperative
  * kernel takes besides (kv heads in fours or twos; fp16 K with 16 < G groups
  * <= 32) that kernel's own: 0 (stream) for a variable-length batch, else a
- * split length.  Same arguments and result as knlp_kv_decode_plan; a caller
+ * split length with at most one block per CU.  Shapes that the per-head kernel
+ * takes as well keep the plan where the rows are many and short (more than
+ * half as many as CUs, up to 24 tiles of 64 or 128 tokens), and the decode
+ * entry points run them on that kernel wherever the splits make more blocks
+ * than CUs.  Same arguments and result as knlp_kv_decode_plan; a caller
  * of either may pass its result to any decode entry point.  The answer is the
  * shape's: where the planes turn out not to lie as that kernel needs them, a
  * stream schedule is run as split-K inside its workspace, with splits sized by

@@ -270,20 +270,44 @@ int32_t knlp_kv_decode_schedule(int32_t num_seqs, int32_t num_kv_heads, int32_t 
   const int parts = coop_extra_parts(num_kv_heads, group, head_size, k_format, k_group_size,
                                      v_format, v_group_size);
   if (parts == 0) return plan;
-  // The plan's rules with this kernel's heads per block: the stream schedule
-  // for a variable-length batch, else one block per CU.
   const int64_t rect = static_cast<int64_t>(num_seqs) * max_context;
   const int64_t total = total_context > 0 ? total_context : rect;
   const bool ragged = total_context > 0 ? 10 * total <= 9 * rect : num_seqs > 1;
-  if (ragged && num_seqs <= kStreamMaxSeqs && max_context <= kStreamMaxContext) return 0;
-  const int heads = k_format == KNLP_KV_FP16 ? 4 : 8 / parts;
-  const int64_t hgroups = num_kv_heads / heads;
+  const int64_t hgroups = num_kv_heads / coop_extra_heads(k_format, parts);
+  const int64_t rows = num_seqs * hgroups, cus = num_cus();
   const int64_t tile = 32LL * parts > 64 ? 32LL * parts : 64;   // whole tiles, multiples of 64
+  const int64_t n = (max_context + tile - 1) / tile;            // tiles of a row
+  // INT4 K and V of one head set run on the per-head kernel too, on the plan's
+  // splits: small blocks, several to a CU, where this kernel has one block per
+  // CU and 6-8 us of start-up to a row.  That one is better for many short
+  // rows, this one for few or long ones.  us per call of lengths up to the one
+  // named, plan / split-K (all lengths equal) / stream:
+  //   12 / 12 heads of 64, 64 x 200 ragged: 14.2 / 16.5 / 18.6
+  //   256 x 500:  42 / - / 46;  700 x 150: 39 / - / 76;  32 x 4000: 58 / 45 / 28
+  //   28 / 4 of 128 in groups of 64, 96 x 1000: 25 / 22 / 33;  128 x 2000: 42 / - / 37
+  //   14 / 2 of 64, 4 x 1000: 10.7 / 10.6 / 13.4;  16 x 9000: 23 / 18.4 / 18
+  const bool per_head = knlp_kv_decode_kernel_kind(num_q_heads, num_kv_heads, head_size, k_format,
+                                                   k_group_size, v_format, v_group_size, 0) == 1;
+  if (ragged && num_seqs <= kStreamMaxSeqs && max_context <= kStreamMaxContext) {
+    if (!per_head) return 0;
+    // (a row's tiles at twice the mean length, where that is known)
+    const int64_t most = total_context > 0
+                             ? std::min(n, (2 * total / num_seqs + tile - 1) / tile) : n;
+    if (most > 24 && rows * n >= cus) return 0;
+    if (most <= 24 && (n > 24 || 2 * rows > cus)) return plan;
+  } else if (per_head && (rows > cus || (2 * rows > cus && n <= 12))) {
+    return plan;
+  }
+  // at most one block per CU: a second round of blocks would double the time
+  // (28 / 4 heads in groups of 64, 48 x 9000 tokens: 288 blocks 95 us, 240 58)
+  if (rows <= cus) {
+    const int64_t ns = cus / rows;
+    return static_cast<int32_t>((n + ns - 1) / ns * tile);
+  }
   // (a batch of more sequences than the stream schedule holds: at least a
   // quarter of the uniform batch's split, as in the plan, since scratch is
   // [num_seqs, hq, ceil(max_context / t)] whatever the lengths)
-  const int64_t t = std::max((total * hgroups + num_cus() - 1) / num_cus(),
-                             (rect * hgroups + num_cus() - 1) / num_cus() / 4);
+  const int64_t t = std::max((total * hgroups + cus - 1) / cus, (rect * hgroups + cus - 1) / cus / 4);
   const int64_t most = (static_cast<int64_t>(max_context) + 63) / 64 * 64;
   return static_cast<int32_t>(std::min(std::max<int64_t>((t + tile - 1) / tile, 1) * tile, most));
 }
@@ -440,9 +464,15 @@ int decode_partial(const void* query, int32_t q_dtype, int64_t q_stride_seq,
   hipStream_t hs = static_cast<hipStream_t>(stream_ptr);
   // (any finite softmax scale: the matrix-core kernels fold a negative one's
   // sign into q and treat 0 as uniform weights)
-  const int extra = coop_extra_supported(a, head_size);
   const bool mfma = kind == 1 && mfma_layout_ok(kp, head_size, block_size) &&
                     mfma_layout_ok(vp, head_size, block_size);
+  int extra = coop_extra_supported(a, head_size);
+  // more blocks than CUs, of which the cooperative kernel runs one per CU at a
+  // time: the per-head kernel where it takes the planes (knlp_kv_decode_schedule)
+  if (extra && mfma && !stream &&
+      static_cast<int64_t>(ns) * num_seqs * (num_kv_heads / coop_extra_heads(kp.format, extra)) >
+          num_cus())
+    extra = 0;
   int32_t* fallback_hdr = nullptr;
   if (stream && !extra && !(mfma && stream_supported(a, head_size))) {
     // Planes only the split schedule takes (fp16 K at D = 64, an odd number of

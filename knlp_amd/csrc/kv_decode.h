@@ -172,6 +172,10 @@ int launch_merge(const float* part_o, const float* part_ml, const int32_t* seq_l
 int coop_extra_parts(int num_kv_heads, int group, int head_size, int k_format, int k_gs,
                      int v_format, int v_gs);
 int coop_extra_supported(const DecodeArgs& a, int head_size);
+// kv heads per block of those instances
+inline int coop_extra_heads(int k_format, int parts) {
+  return k_format == KNLP_KV_FP16 ? 4 : 8 / parts;
+}
 int launch_decode_extra(const DecodeArgs& a, int head_size, int parts, hipStream_t stream);
 // launches the stream schedule (one block per CU) when a.stream is set; false
 // if this shape has no cooperative kernel (the stream schedule needs it)

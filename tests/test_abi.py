@@ -339,6 +339,38 @@ def test_schedule_is_the_plan_where_no_layout_fits_the_narrow_kernels():
         assert L.knlp_kv_decode_schedule(8, hkv, hq, d, 4096, 0, *fmt) == 0
 
 
+@pytest.mark.parametrize("hq,hkv,d,gs,rows,tile", [(12, 12, 64, 32, 3, 64), (14, 2, 64, 32, 1, 128),
+                                                    (16, 4, 128, 32, 1, 64), (28, 4, 128, 64, 1, 64)])
+def test_schedule_leaves_many_short_rows_to_the_per_head_kernel(hq, hkv, d, gs, rows, tile):
+    """Shapes that the per-head kernel takes too (256 CUs).  Many short rows: the
+    plan's splits, and more blocks of the cooperative kernel than CUs, which is
+    what the decode goes by; else at most one block per CU, or the stream
+    schedule for long rows of unequal lengths."""
+    L = _lib.lib()
+    fmt = (_lib.KV_INT4_ASYM, gs, _lib.KV_INT4_ASYM, gs)
+
+    def both(S, mc, total):
+        a = (S, hkv, hq, d, mc, total, *fmt)
+        return L.knlp_kv_decode_schedule(*a), L.knlp_kv_decode_plan(*a)
+
+    def blocks(S, mc, split):
+        return S * rows * -(-mc // split)
+    for S, mc in ((256, 80), (512, 200), (700, 160), (1000, 512), (1200, 128)):
+        for total in (0, S * mc // 2, S * mc):
+            got, plan = both(S, mc, total)
+            assert got == plan and blocks(S, mc, plan) > 256, (S, mc, total)
+    # short rows in a wide table, their total known
+    got, plan = both(300, 65536, 300 * 300)
+    assert got == plan
+    for S, mc in ((1, 1024), (4, 512), (16, 4096), (48, 9008), (85, 2048)):
+        got, plan = both(S, mc, S * mc)
+        assert got % tile == 0 and blocks(S, mc, got) <= 256, (S, mc, got)
+        # ... as many blocks as that allows
+        assert got == tile or blocks(S, mc, got - tile) > 256 or -(-mc // got) == -(-mc // (got - tile))
+    assert both(64 // rows, 16384, 0)[0] == 0 and both(200, 8192, 0)[0] == 0
+    assert 0 < both(4, 1024, 0)[0] and blocks(4, 1024, both(4, 1024, 0)[0]) <= 256
+
+
 def _rows_plane(fmt, hkv, d, gs, page=16, room=0, apart=1):
     """A plane of hkv heads, cut out of one of hkv + room, every `apart`-th one."""
     row = d if fmt in (_lib.KV_FP16, _lib.KV_INT8_SYM) else d // 2
