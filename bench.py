@@ -335,8 +335,7 @@ CPU_PASS_BUDGET_S = 1.6
 def time_cpu_baseline(cfg, q_cpu, kc: Caches, vc: Caches, bt, seq_lens, bs):
     """The reference's CPU path (the oracle's dequantise -> repeat_interleave
     -> SDPA in torch fp32, scripts/v35_h100_bench.py:376-387) on the host
-    cores, timed per BASELINE's CPU plan: all the CPUs this process may use,
-    the median of 10 timed passes after 5 warm ones.  A pass covers the whole
+    cores, timed with all the CPUs this process may use: the median of 10 timed passes after 5 warm ones.  A pass covers the whole
     step when one step fits about 1.6 s of CPU time (config 2: 8 sequences,
     about 1.5 s on 16 cores), otherwise the first sequences (longest first for
     variable lengths) that do, so the baseline costs at most about 25 s; the

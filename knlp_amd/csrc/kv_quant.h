@@ -18,7 +18,7 @@
 // with IEEE division on the CPU: every mantissa of the scale, v_rcp results up
 // to 2 ulp off, every rounding threshold k - 1/2 (k = 1 .. 128) and x within
 // 4 ulps of it (4.8e10 cases) give the same code, and the constant divisors
-// the same quotient for every mantissa.  Both are exact in the exponent while
+// the same quotient for every mantissa (a sample of it: test_quotients.py).  Both are exact in the exponent while
 // nothing over- or underflows, which `safe` tests for (else the wave divides).
 // An IEEE division is about 11 VALU operations, the step 3.
 #pragma once

@@ -26,7 +26,7 @@ def kv_bytes(c, kfmt=None, vfmt=None):
     return total - qo - bt, sl
 
 
-# K + V bytes per decode step at the BASELINE shapes, worked out by hand:
+# K + V bytes per decode step at the benchmark shapes, worked out by hand:
 #   1: 1 seq x 1024 tok x 12 heads x 2 x (32 + 2*2*2)            =       983,040
 #   2: 8 x 32768 x 8 x 2 x (64 + 4*2*2)                          =   335,544,320
 #   4: 1 x 393216 x 8 x 2 x (64 + 2*2*2)                         =   452,984,832

@@ -1,4 +1,4 @@
-"""The BASELINE configurations 2-5 at their full size on the GPU.
+"""The benchmark configurations 2-5 at their full size on the GPU.
 
 The oracle cannot decode whole batches of these sizes in the test budget, so
 the checks are the size-independent properties the reference's own at-shape

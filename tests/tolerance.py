@@ -1,6 +1,6 @@
 """The decode parity bar, and a record of the error each GPU case achieved.
 
-Bar (BASELINE north_star): max |gpu - oracle| <= 2e-3 against the oracle's
+Bar: max |gpu - oracle| <= 2e-3 against the oracle's
 fp32 dequantise -> SDPA result before output rounding.  Only the GPU side is
 rounded to the output type there, so above |oracle| = 2 the bar adds what
 that one rounding can contribute:
