@@ -168,17 +168,22 @@ def prefill_supported(query, key, value, out, scale) -> bool:
     if not (query.is_cuda and query.dtype in _SRC_DTYPES and query.dim() == 3 and
             query.shape[2] in (64, 128) and (scale is None or abs(scale) < 2.0 ** 127)):
         return False
+    d = query.shape[2]
+    spans = []                             # first byte and the one past the last
     for t in (query, key, value, out):
-        if (t.dim() != 3 or t.dtype != query.dtype or t.device != query.device or
-                t.shape[2] != query.shape[2] or t.stride(2) != 1 or t.stride(0) % 8 or
-                t.stride(1) % 8 or t.data_ptr() % 16):
+        if t.dim() != 3 or t.dtype != query.dtype or t.device != query.device:
             return False
-    if not all(query.shape[2] <= t.stride(0) < 1 << 24 for t in (key, value)):
+        (n, h, last), (st, sh, one), p = t.shape, t.stride(), t.data_ptr()
+        if last != d or one != 1 or st % 8 or sh % 8 or p % 16:
+            return False
+        spans.append((p, p + 2 * ((n - 1) * st + (h - 1) * sh + d)))
+    if not all(d <= t.stride(0) < 1 << 24 for t in (key, value)):
         return False                       # repeated or overlapping rows
-    if any(_same_storage(out, t) for t in (key, value)):
+    first, end = spans[3]
+    if any(first < e and s < end for s, e in spans[1:3]):
         return False
-    if _same_storage(out, query) and (out.data_ptr() != query.data_ptr() or
-                                      out.stride() != query.stride()):
+    if first < spans[0][1] and spans[0][0] < end and (first != spans[0][0] or
+                                                      out.stride() != query.stride()):
         return False                       # (in place: a block reads only the rows it writes)
     return (out.shape[1] == query.shape[1] and key.shape[1] == value.shape[1] > 0 and
             query.shape[1] % key.shape[1] == 0)
