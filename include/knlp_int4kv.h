@@ -150,7 +150,7 @@ int32_t knlp_kv_decode_plan(int32_t num_seqs, int32_t num_kv_heads,
  * <= 32) that kernel's own: 0 (stream) for a variable-length batch, else a
  * split length with at most one block per CU.  Shapes that the per-head kernel
  * takes as well keep the plan where the rows are many and short (more than
- * half as many as CUs, up to 24 tiles of 64 or 128 tokens), and the decode
+ * half as many as CUs, max_context up to 24 tiles of 64 or 128 tokens), and the decode
  * entry points run them on that kernel wherever the splits make more blocks
  * than CUs.  Same arguments and result as knlp_kv_decode_plan; a caller
  * of either may pass its result to any decode entry point.  The answer is the

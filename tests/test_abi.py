@@ -359,9 +359,10 @@ def test_schedule_leaves_many_short_rows_to_the_per_head_kernel(hq, hkv, d, gs, 
         for total in (0, S * mc // 2, S * mc):
             got, plan = both(S, mc, total)
             assert got == plan and blocks(S, mc, plan) > 256, (S, mc, total)
-    # short rows in a wide table, their total known
-    got, plan = both(300, 65536, 300 * 300)
-    assert got == plan
+    # short rows in a wide table: whatever their total, the stream schedule (the
+    # plan's splits would be nearly all empty)
+    for S in (16, 100, 300):
+        assert both(S, 65536, S * 300)[0] == 0
     for S, mc in ((1, 1024), (4, 512), (16, 4096), (48, 9008), (85, 2048)):
         got, plan = both(S, mc, S * mc)
         assert got % tile == 0 and blocks(S, mc, got) <= 256, (S, mc, got)
